@@ -253,6 +253,7 @@ void tile_gemm_kernel(GemmGroup gp) {
   }
   barrier();
   fetch_raw(0);
+  barrier();   // block 0's weights are out of LDS before group 0's first step writes W(2) there
   auto dequant = [&]() __attribute__((always_inline)) {
     const bool fast = (bool)__all(one_rounding_exact<QBITS>(sh, zh));
 #pragma unroll
@@ -269,8 +270,8 @@ void tile_gemm_kernel(GemmGroup gp) {
   // weights and scales of block kb + 1 out of LDS, X(kb + 1) and W(kb + 2) into LDS, the
   // loads of X(kb + 3) and W(kb + 4).  Dequantisation phase: the fragments of kb + 1.
   // Group 0 multiplies block kb in interval 2 kb, group 1 in interval 2 kb + 1; a stage is
-  // written there after its last read (X(kb - 1), W(kb): intervals 2 kb - 2 and 2 kb - 1)
-  // and before its next (2 kb + 2).
+  // written there after its last read (X(kb - 1), W(kb): intervals 2 kb - 2 and 2 kb - 1, for
+  // W(0) the prologue's, which its own barrier ends) and before its next (2 kb + 2).
   auto step = [&](int kb, auto cur_c) __attribute__((always_inline)) {
     constexpr int CUR = decltype(cur_c)::value, NXT = CUR ^ 1;
     constexpr int NOPS = 4 * MT, AHEAD = TG_AHEAD, RING = AHEAD + 1, COPIES = S::XCH + S::WCH;
