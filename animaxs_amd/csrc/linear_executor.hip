@@ -154,11 +154,12 @@ bool LinearExecutor::encode_group(anima_buffer input, const anima_qweight* const
                (i == 0 || (w.storage == storage && ps[i].K == ps[0].K));
     storage = w.storage;
     if (!together) continue;
-    if (epi && epi[i].epilogue == GEMM_QK_NORM) ps[i].epilogue = GEMM_QK_NORM;
-    const bool small = tile_preferred(ps[i], storage);
+    const bool small = tile_preferred(ps[i], storage), norm = epi && epi[i].epilogue == GEMM_QK_NORM;
     small_tiles += small ? 1 : 0;
     tiles += pingpong_tiles(ps[i]);
-    same_bits = same_bits && (count == 1 || (small ? tile_ksplit(ps[i]) == 1 : !pingpong_msplit(ps[i], storage))) &&
+    // Alone, a linear keeps its split or its M-split form here; split sums take no Q/K norm.
+    same_bits = same_bits && (small ? (count == 1 && !norm) || tile_ksplit(ps[i]) == 1
+                                    : count == 1 || !pingpong_msplit(ps[i], storage)) &&
                 (!small || tile_shape(ps[i]) == tile_shape(ps[0]));
   }
   // Small tiles pay several rounds where one of 128 x 256 tiles would do.

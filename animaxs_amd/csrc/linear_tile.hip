@@ -432,7 +432,6 @@ bool tile_takes_norm(const GemmParams& p) { return TG_TN[tile_shape(p)] % 128 ==
 // none): W4 M=109 N=128 K=5696 26.4 -> 16.9, W8 M=191 N=752 K=6016 28.2 -> 18.6, W4 M=3153
 // N=160 K=7232 50.4 -> 35.7, W8 M=1451 N=1200 K=4672 87 (before this kernel) -> 38.9.
 int tile_ksplit(const GemmParams& p) {
-  if (p.epilogue == GEMM_QK_NORM) return 1;
   const int shape = tile_shape(p), min_blocks = shape ? 4 : 8;
   const int64_t tiles = tile_count(p, shape);
   for (int k = 8; k > 1; --k) {
