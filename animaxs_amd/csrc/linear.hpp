@@ -170,6 +170,10 @@ void launch_smallm(const GemmParams& p, int storage, hipStream_t stream);
 // p.part = [slices][M][N] fp32 and p.ksplit = slices; launch_smallm_splitk adds the
 // slices in order (launch_splitk_epilogue) into p.y.
 int smallm_splitk_slices(const GemmParams& p, int storage);
+// Whether a plain linear runs one of the two small-M kernels.
+inline bool smallm_preferred(const GemmParams& p, int storage) {
+  return smallm_supported(p, storage) || smallm_splitk_slices(p, storage) > 0;
+}
 void launch_smallm_splitk(const GemmParams& p, int storage, hipStream_t stream);
 // The splits' sum in order, rounded once, through p's output stage (not GEMM_QK_NORM).
 void launch_splitk_epilogue(const GemmParams& p, hipStream_t stream);

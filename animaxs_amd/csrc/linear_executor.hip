@@ -150,7 +150,7 @@ bool LinearExecutor::encode_group(anima_buffer input, const anima_qweight* const
     // Up to 64 rows a single linear streams its weights in another kernel; one launch of the
     // small tiles is still faster than two or three of those (encoder layer of 8 / 40 / 62
     // tokens, Q, K and V together: 57.5 -> 48.5, 66.4 -> 52.8, 72.4 -> 56.2 us).
-    together = together && (one_launch || !smallm_supported(ps[i], w.storage)) && pingpong_supported(ps[i], w.storage) &&
+    together = together && (one_launch || !smallm_preferred(ps[i], w.storage)) && pingpong_supported(ps[i], w.storage) &&
                (i == 0 || (w.storage == storage && ps[i].K == ps[0].K));
     storage = w.storage;
     if (!together) continue;
@@ -206,7 +206,7 @@ bool LinearExecutor::encode_fused(anima_buffer input, int64_t input_offset, cons
     fail(ANIMA_E_INVALID_SHAPE, "invalid LinearExecutor shape or offset");
   const QWeightView w = validate_weight(weight, "LinearExecutor");
   GemmParams p = prepare(input, input_offset, w, output, output_offset, input_rows);
-  if (cfg_.backend != ANIMA_LINEAR_BACKEND_AUTO || smallm_supported(p, w.storage) || !pingpong_supported(p, w.storage))
+  if (cfg_.backend != ANIMA_LINEAR_BACKEND_AUTO || smallm_preferred(p, w.storage) || !pingpong_supported(p, w.storage))
     return false;
   p.epilogue = epilogue;
   p.residual = residual;
