@@ -553,9 +553,7 @@ __global__ __launch_bounds__(PRO_D128_THREADS) void qk_prologue_d128_kernel(Prol
     for (int i = 0; i < 8; ++i) rrow[i] = blk[8 * i];
 #pragma unroll
     for (int i = 0; i < 8; ++i) lds[8 * i + (sub ^ i)] = rrow[i];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_exchange();
 #pragma unroll
     for (int i = 0; i < 8; ++i) rrow[i] = lds[8 * sub + (i ^ sub)];
   }

@@ -113,13 +113,16 @@ void flash_attention_short_kernel(FlashParams p) {
       for (int i = 0; i < NP; ++i) x.r[i] = t[2 * LPR * (i >> 1) + (i & 1)];
     }
   };
-  // Norm and RoPE in fp32, times mul, one rounding, in LDS row dst.  The lower table row is
-  // [sin, cos] for K and taken as [-(-sin), cos] for Q, as the Q prologue of the other flash
-  // kernels and the K prologue kernel read it.
-  auto store_row = [&](const Row& x, const half_t* w, const float* rope, bool q, float mul, half_t* dst)
-      __attribute__((always_inline)) {
+  auto put_row = [&](const Row& x, half_t* dst) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < XP; ++i) *reinterpret_cast<u32x4*>(dst + 8 * (sub + LPR * i)) = x.x[i];
+  };
+  // Norm and RoPE in fp32, times mul, one rounding, in LDS row dst, which other lanes of the
+  // row put there (wave_lds_exchange between).  The lower table row is
+  // [sin, cos] for K and taken as [-(-sin), cos] for Q, as the Q prologue of the other flash
+  // kernels and the K prologue kernel read it.
+  auto norm_row = [&](const Row& x, const half_t* w, const float* rope, bool q, float mul, half_t* dst)
+      __attribute__((always_inline)) {
     if (!w && !rope && !q) return;
     float a[NP], c[NP];
 #pragma unroll
@@ -183,14 +186,19 @@ void flash_attention_short_kernel(FlashParams p) {
   };
   // rows: key rows of the chunk in use.  K rows past them are never multiplied into a score
   // that is kept, V rows must read as zeros up to the next multiple of 32.
-  auto store_chunk = [&](int rows) __attribute__((always_inline)) {
+  auto put_chunk = [&](int rows) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < KP; ++i)
-      if (RPP * (FS_WAVES * i + wave) < rows) store_row(kr[i], p.k_norm_w ? NW + D : nullptr, p.k_rope, false, 1.f,
-                Ks + (RPP * (FS_WAVES * i + wave) + prow) * KROW);
+      if (RPP * (FS_WAVES * i + wave) < rows) put_row(kr[i], Ks + (RPP * (FS_WAVES * i + wave) + prow) * KROW);
 #pragma unroll
     for (int i = 0; i < VP; ++i)
       *reinterpret_cast<u32x4*>(Vs + (tid / VCH + FS_NT / VCH * i) * VROW + 8 * (tid % VCH)) = vr[i];
+  };
+  auto norm_chunk = [&](int rows) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < KP; ++i)
+      if (RPP * (FS_WAVES * i + wave) < rows) norm_row(kr[i], p.k_norm_w ? NW + D : nullptr, p.k_rope, false, 1.f,
+                Ks + (RPP * (FS_WAVES * i + wave) + prow) * KROW);
   };
 
   {
@@ -209,9 +217,12 @@ void flash_attention_short_kernel(FlashParams p) {
     load_chunk(0);
     if (nw) *reinterpret_cast<half8v*>(NW + 8 * lane) = nv;
     barrier();
-    if (q_wave)
-      store_row(qr, p.q_norm_w ? NW : nullptr, p.rope, true, p.scale_log2, Qs + (RPP * wave + prow) * KROW);
-    store_chunk(kend);
+    half_t* const q_row = Qs + (RPP * wave + prow) * KROW;
+    if (q_wave) put_row(qr, q_row);
+    put_chunk(kend);
+    wave_lds_exchange();
+    if (q_wave) norm_row(qr, p.q_norm_w ? NW : nullptr, p.rope, true, p.scale_log2, q_row);
+    norm_chunk(kend);
   }
   barrier();
 
@@ -306,7 +317,9 @@ void flash_attention_short_kernel(FlashParams p) {
     }
     if (ch + 1 < nchunk) {
       barrier();   // every read of this chunk's K and V rows done
-      store_chunk(left - FS_BK);
+      put_chunk(left - FS_BK);
+      wave_lds_exchange();
+      norm_chunk(left - FS_BK);
       barrier();
     }
   }
