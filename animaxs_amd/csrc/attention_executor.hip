@@ -263,12 +263,17 @@ void AttentionExecutor::encode_impl(const anima_attention_args& a, bool no_alloc
     p.rope = rope_q;
   }
   // Short sequences: one launch with both prologues fused, in place of the K prologue and
-  // the 256-row kernel.  Asked on the strides of the caller's rows, which it reads.  Output
-  // rows over the key rows are fine only behind a prologue that copied the keys.
-  const bool over_keys = reinterpret_cast<const char*>(op) < reinterpret_cast<const char*>(kp) + k_bytes &&
-                         reinterpret_cast<const char*>(kp) < reinterpret_cast<const char*>(op) + q_bytes;
+  // the 256-row kernel.  Asked on the strides of the caller's rows, which it reads.  Its
+  // workgroups finish in any order over 32-row tiles, so output rows may lie only over the very
+  // query rows; over other inputs the launches stay as they were (a K prologue copies the keys,
+  // and up to 256 queries one workgroup reads all of a head before it writes).
+  auto over = [&](const half_t* in, int64_t bytes) {
+    const uintptr_t i = reinterpret_cast<uintptr_t>(in), o = reinterpret_cast<uintptr_t>(op);
+    return o < i + bytes && i < o + q_bytes;
+  };
+  const bool over_inputs = over(kp, k_bytes) || over(vp, k_bytes) || (op != qp && over(qp, q_bytes));
   bool use_short = false;
-  if (use_flash && cfg_.flash_rows == 0 && !need_q_pro && !(need_k_pro && over_keys) && (!k_norm || aligned16(k_norm)) &&
+  if (use_flash && cfg_.flash_rows == 0 && !need_q_pro && !over_inputs && (!k_norm || aligned16(k_norm)) &&
       (!rope_k || aligned16(rope_k))) {
     FlashParams ps = p;
     ps.k_tok = k_in_tok; ps.k_head = k_in_head; ps.k_batch = k_in_batch;

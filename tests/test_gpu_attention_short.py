@@ -107,3 +107,27 @@ def test_output_over_the_keys(ctx):
         prologue=QKPrologue(None, dev(kw), 1e-6, None, 0, False, False))
     ref = oatt.sdpa(q, oatt.qk_prologue(k, kw, 1e-6, None), v)
     assert_attention_close(kd.float().cpu(), ref)
+
+
+@pytest.mark.parametrize("where", ["key", "value", "query", "query shifted"])
+@pytest.mark.parametrize("S,D", [(40, 64), (70, 128), (256, 128)])
+def test_output_over_an_input(ctx, where, S, D):
+    """Up to 256 queries the output may take an input's place, whatever kernel runs: the bits of
+    the 256-row kernel where it does, and the query's own rows in the short kernel too."""
+    g = torch.Generator().manual_seed(S)
+    x = {n: torch.randn(S, 1, D, generator=g).half() for n in ("query", "key", "value")}
+    kw = dict(heads=1, query_count=S, key_count=S, head_dim=D)
+    want = torch.empty(S, 1, D, dtype=torch.float16, device="cuda")
+    print(f"OVER {where} S={S} D={D}", flush=True)
+    rows = 0 if where == "query" else 256
+    AttentionExecutor(ctx, layout=("tokenMajor", D), flash_rows=rows).execute(
+        **{n: dev(t) for n, t in x.items()}, output=want, **kw)
+    d = {n: dev(t) for n, t in x.items()}
+    if where == "query shifted":   # eight rows into the buffer that holds the query rows
+        d["query"] = dev(torch.cat([x["query"], torch.zeros(8, 1, D, dtype=torch.float16)]))
+        AttentionExecutor(ctx, layout=("tokenMajor", D)).execute(**d, output=d["query"], output_offset=16 * D, **kw)
+        got = d["query"][8:]
+    else:
+        AttentionExecutor(ctx, layout=("tokenMajor", D)).execute(**d, output=d[where], **kw)
+        got = d[where]
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
