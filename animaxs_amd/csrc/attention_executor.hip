@@ -290,8 +290,9 @@ void AttentionExecutor::encode_impl(const anima_attention_args& a, bool no_alloc
     part = splits > 1 ? round_up(flash_split_bytes(p, (int)D, (int)B, splits), 256) : 0;
   };
   plan_splits(1);
-  // The static scratch holds what it held before fine splits.
-  if (no_alloc && k_ws + q_ws + part > NOALLOC_SCRATCH_BYTES) plan_splits(0);
+  // Fine splits only where the static scratch holds them: both entry points take one plan, so
+  // their results are the same, and the scratch holds what it held without fine splits.
+  if (k_ws + q_ws + part > NOALLOC_SCRATCH_BYTES) plan_splits(0);
 
   DeviceGuard guard(ctx_);
   hipStream_t stream = ctx_->stream;

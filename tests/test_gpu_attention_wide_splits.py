@@ -63,3 +63,20 @@ def test_wide_noalloc_beyond_its_scratch_takes_fewer_splits(ctx):
     ref = oatt.sdpa(tm[0], oatt.qk_prologue(tm[1], kw, 1e-6, None), tm[2])
     for o in outs:
         assert_attention_close(o.permute(0, 2, 1, 3), ref)
+
+
+def test_wide_noalloc_equals_encode_beyond_its_scratch(ctx):
+    """The same plan, and so the same bits, also where fine splits would exceed the scratch."""
+    B, Sq, Sk = 64, 128, 1000
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (dev(torch.randn(B, 1, n, D, generator=g).half()) for n in (Sq, Sk, Sk))
+    kw = dev((0.8 + 0.4 * torch.rand(D, generator=g)).half())
+    ex = AttentionExecutor(ctx, layout="headMajor")
+    args = dict(query=q, key=k, value=v, heads=1, query_count=Sq, key_count=Sk, head_dim=D, batch=B,
+                prologue=QKPrologue(None, kw, 1e-6, None, 0, False, False))
+    outs = [torch.full((B, 1, Sq, D), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2)]
+    print("WIDE scratch limit", flush=True)
+    ex.encode(output=outs[0], **args)
+    ex.encode_noalloc(output=outs[1], **args)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
