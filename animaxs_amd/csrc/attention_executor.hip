@@ -296,6 +296,8 @@ void AttentionExecutor::encode_impl(const anima_attention_args& a, bool no_alloc
 
   DeviceGuard guard(ctx_);
   hipStream_t stream = ctx_->stream;
+  // A first call under capture cannot allocate for them either.
+  if (!no_alloc && !split_ws_.available(part, stream)) plan_splits(0);
   char* ws = nullptr;
   char* pw = nullptr;
   if (no_alloc) {

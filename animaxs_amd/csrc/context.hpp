@@ -49,9 +49,17 @@ class Workspace {
     capacity_ = cap;
     return ptr_;
   }
+  // Whether get(bytes, stream) can serve: nothing can be allocated while the stream is captured.
+  bool available(int64_t bytes, hipStream_t stream) const { return bytes <= capacity_ || !capturing(stream); }
   int64_t capacity() const { return capacity_; }
 
  private:
+  static bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // the null stream while another one is captured
+    return true;
+  }
   void release() {
     if (ptr_) (void)hipFree(ptr_);
     ptr_ = nullptr;

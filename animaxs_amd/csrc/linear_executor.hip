@@ -82,8 +82,10 @@ void LinearExecutor::plan_tile_splits(GemmParams& p, int storage, hipStream_t st
   if (!tile_preferred(p, storage)) return;
   const int ks = tile_ksplit(p);
   if (ks == 1) return;
+  const int64_t bytes = checked_product({(int64_t)ks, p.M, p.N, 4}, "LinearExecutor");
+  if (!ws_.available(bytes, stream)) return;   // a first call under capture runs unsplit
   p.ksplit = ks;
-  p.part = static_cast<float*>(ws_.get(checked_product({(int64_t)ks, p.M, p.N, 4}, "LinearExecutor"), stream));
+  p.part = static_cast<float*>(ws_.get(bytes, stream));
 }
 
 void LinearExecutor::encode(anima_buffer input, int64_t input_offset, const anima_qweight& weight,
@@ -115,10 +117,10 @@ void LinearExecutor::encode(anima_buffer input, int64_t input_offset, const anim
     return;
   }
   const int slices = cfg_.backend == ANIMA_LINEAR_BACKEND_AUTO ? smallm_splitk_slices(p, w.storage) : 0;
-  if (slices > 0) {
+  const int64_t part = slices > 1 ? checked_product({(int64_t)slices, p.M, p.N, 4}, "LinearExecutor") : 0;
+  if (slices > 0 && ws_.available(part, stream)) {
     p.ksplit = slices;
-    if (slices > 1)
-      p.part = static_cast<float*>(ws_.get(checked_product({(int64_t)slices, p.M, p.N, 4}, "LinearExecutor"), stream));
+    if (slices > 1) p.part = static_cast<float*>(ws_.get(part, stream));
     launch_smallm_splitk(p, w.storage, stream);
     return;
   }
