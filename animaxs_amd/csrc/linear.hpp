@@ -133,6 +133,12 @@ void launch_pingpong(const GemmParams& p, int storage, hipStream_t stream);
 // Its 128 x 256 tiles, and how many fill half the chip.
 inline int64_t pingpong_tiles(const GemmParams& p) { return (int64_t)((p.M + 127) / 128) * ((p.N + 255) / 256); }
 constexpr int64_t PG_FILL = 128;
+// Output rows over the input's: right where one workgroup reads all of X before it writes, as in
+// a ping-pong launch of one tile.  Such a linear is left to that kernel.
+inline bool single_tile_over_input(const GemmParams& p) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(p.x), y = reinterpret_cast<uintptr_t>(p.y);
+  return pingpong_tiles(p) == 1 && y < x + (int64_t)p.M * p.K * 2 && x < y + (int64_t)p.M * p.N * 2;
+}
 // count (1..PG_GROUP) ping-pong GEMMs sharing K and storage in one launch.
 void launch_pingpong_group(const GemmParams* ps, int count, int storage, hipStream_t stream);
 // Whether a single launch of p runs the M-split form (256-row tiles, no K split between

@@ -486,6 +486,7 @@ static bool smallm_fits(int M, int K) {
 bool smallm_supported(const GemmParams& p, int storage) {
   const int whole = storage == ANIMA_STORAGE_FP16 ? SM_CHUNK : SM_CHUNK / 2;
   if (p.M < 1 || p.M > SMALLM_MAX_ROWS || p.K < 1 || p.K % whole != 0 || !aligned16(p.x) || !aligned16(p.w)) return false;
+  if (p.K % SM_CHUNK != 0 && single_tile_over_input(p)) return false;
   if ((int64_t)p.M * p.K * 2 > 0x7fffffff) return false;   // X is addressed with 32-bit buffer offsets
   if (storage == ANIMA_STORAGE_FP16) return p.row_stride % 8 == 0 && smallm_fits<ANIMA_STORAGE_FP16>(p.M, p.K);
   if (p.row_stride % 16 != 0) return false;
@@ -712,7 +713,7 @@ static int splitk_chunks(const GemmParams& p, int storage) {
   // 17.4 -> 14.9 us; M=16 K=4096 ties and M=32 N=4096 K=2048 is 5 % slower split.
   if (p.N >= 32 * 256 || (p.M <= 32 && (int64_t)p.M * p.K < 131072)) return 0;
   if (p.M < 1 || p.M > SMALLM_MAX_ROWS || p.K < 1 || p.K % (SM_CHUNK / 2) != 0 || !aligned16(p.x) || !aligned16(p.w) ||
-      p.row_stride % 16 != 0 || (int64_t)p.M * p.K * 2 > 0x7fffffff)
+      p.row_stride % 16 != 0 || (int64_t)p.M * p.K * 2 > 0x7fffffff || (p.K % SM_CHUNK != 0 && single_tile_over_input(p)))
     return 0;
   const int mb = (p.M + 15) / 16, nch = (p.K + SM_CHUNK - 1) / SM_CHUNK;
   const int64_t rgroups = (p.N + SK_ROWS - 1) / SK_ROWS;

@@ -414,7 +414,7 @@ static int64_t tile_count(const GemmParams& p, int shape) {
 // M=4096 N=1024 K=2048 33.6-35 / 29-31.5; at 96 M=1024 N=3072 K=1024 18.7-20.2 / 18.7-20.0; at
 // 64 M=1024 N=2048 K=2048 17.3 / 29.4.
 bool tile_preferred(const GemmParams& p, int storage) {
-  if (!pingpong_supported(p, storage)) return false;
+  if (!pingpong_supported(p, storage) || single_tile_over_input(p)) return false;
   return pingpong_tiles(p) < PG_FILL;
 }
 
