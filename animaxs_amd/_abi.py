@@ -274,8 +274,8 @@ def _bind_calls(lib: C.CDLL) -> None:
     try:
         from . import _calls
     except ImportError as e:
-        raise RuntimeError("animaxs_amd/_calls.so is missing or does not load: build it with "
-                           "`python -m animaxs_amd.build` (there is no fallback)") from e
+        raise RuntimeError("the native call module animaxs_amd/_calls is missing for this interpreter or does not "
+                           "load: build it with `python -m animaxs_amd.build` (there is no fallback)") from e
     from . import executors as ex
     names = ("anima_attention_encode", "anima_attention_encode_noalloc", "anima_attention_execute",
              "anima_linear_encode", "anima_linear_execute", "anima_matvec_encode")

@@ -3,8 +3,9 @@
 ``python -m animaxs_amd.build`` (or ``animaxs_amd.build.build()``) compiles every
 ``csrc/*.hip`` with ``hipcc --offload-arch=gfx950`` and every ``csrc/*.cpp`` with
 ``g++``, then links ``animaxs_amd/libanima_hip.so``; ``csrc/python/calls.cpp`` becomes the
-CPython module ``animaxs_amd/_calls.so``.  Packed-FP32 instruction
-selection is disabled for all device code.
+CPython module ``animaxs_amd/_calls`` under the interpreter's own extension suffix, so that
+another interpreter does not load it.  Packed-FP32 instruction selection is disabled for all
+device code.
 """
 
 from __future__ import annotations
@@ -22,7 +23,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 INCLUDE = ROOT / "include"
 OUT = PKG / "libanima_hip.so"
-CALLS = PKG / "_calls.so"
+CALLS = PKG / ("_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 OBJ = PKG / "_build"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -52,10 +53,11 @@ def _compile(src: Path) -> Path:
 
 
 def _build_calls() -> None:
-    tmp = CALLS.with_suffix(".so.tmp")
+    tmp = CALLS.with_name(CALLS.name + ".tmp")
     _run([shutil.which("g++") or "g++", "-shared", str(CSRC / "python" / "calls.cpp"), "-o", str(tmp), *CXX_FLAGS,
           f"-I{sysconfig.get_paths()['include']}"])
     os.replace(tmp, CALLS)
+    (PKG / "_calls.so").unlink(missing_ok=True)   # any interpreter would load an untagged one
 
 
 def build(verbose: bool = True, jobs: int | None = None) -> Path:

@@ -135,3 +135,11 @@ def test_linear_and_matvec(seen):
         handle = C.c_void_p(64)
     E.LinearExecutor.encode_matvec(Ctx, w, (80, 96), (112, 128), 4, 8)
     assert seen.calls[-1] == ("mv", 64, fields(w.to_c()), {"ptr": 80, "length": 96}, 4, {"ptr": 112, "length": 128}, 8)
+
+
+def test_the_module_carries_this_interpreters_tag():
+    """An untagged module would load under any interpreter, whatever ABI it was compiled for."""
+    import sysconfig
+    from animaxs_amd import _calls, build
+    assert _calls.__file__.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+    assert not (build.PKG / "_calls.so").exists()
