@@ -65,6 +65,7 @@ __device__ __forceinline__ void dq_w8_16(const u32x4 raw, float s, float z, half
 // half loads -> quads: W8 M=265 17.7 -> 11.1 us, M=1995 18.9 -> 12.3, W4 M=4096 19.5 -> 14.8.
 template <int STORAGE, bool FAST, bool QUAD = false>
 __global__ __launch_bounds__(G_NT, 1) void gemm_kernel(GemmParams p, int vec_store) {
+  static_assert(!QUAD || (!FAST && STORAGE != ANIMA_STORAGE_FP16), "quads of packed weights");
   __shared__ __attribute__((aligned(16))) half_t Xs[2][G_BM * G_BK];
   __shared__ __attribute__((aligned(16))) half_t Ws[2][G_BN * G_BK];
   constexpr int XL = G_BM * G_BK / 8 / G_NT;      // 8 X chunks per thread
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_kernel(GemmParams p, int vec_sto
         else if (STORAGE == ANIMA_STORAGE_W8) src = p.w + (int64_t)n * p.row_stride + kbase + part * 16;
         else src = p.w + ((int64_t)n * p.row_stride + kbase + part * 8) * 2;
         wr[r] = *reinterpret_cast<const u32x4*>(src);
-      } else if (QUAD && STORAGE != ANIMA_STORAGE_FP16) {
+      } else if (QUAD) {
         // Whole quads inside the row; what lies past K is zeroed after dequant (store_tile).
         constexpr int QB = STORAGE == ANIMA_STORAGE_W4 ? 2 : 4;   // bytes of a quad
         const int wbytes = (int)((int64_t)(p.N - 1) * p.row_stride) + p.K / 4 * QB;
@@ -474,22 +475,27 @@ __global__ __launch_bounds__(256) void matvec_kernel(MatvecParams p) {
 // ===========================================================================
 // Launchers.
 // ===========================================================================
-// Rows whose quads of K load whole and whose tensors a 32-bit offset reaches (QUAD).
+// W4/W8 rows whose quads of K load whole and whose tensors a 32-bit offset reaches (QUAD).
 static bool gemm_quad(const GemmParams& p, int storage) {
   const int align = storage == ANIMA_STORAGE_W4 ? 2 : 4;
-  return storage != ANIMA_STORAGE_FP16 && p.K % 4 == 0 && aligned8(p.x) && p.row_stride % align == 0 &&
+  return p.K % 4 == 0 && aligned8(p.x) && p.row_stride % align == 0 &&
          reinterpret_cast<uintptr_t>(p.w) % align == 0 && (int64_t)p.M * p.K * 2 <= 0x7fffffff &&
          (int64_t)p.N * p.row_stride <= 0x7fffffff;
 }
 
 template <int S>
 static void launch_gemm_t(const GemmParams& p, bool fast, int vec, dim3 grid, hipStream_t stream) {
-  if (fast)
+  if (fast) {
     hipLaunchKernelGGL((gemm_kernel<S, true>), grid, dim3(G_NT), 0, stream, p, vec);
-  else if (gemm_quad(p, S))
-    hipLaunchKernelGGL((gemm_kernel<S, false, true>), grid, dim3(G_NT), 0, stream, p, vec);
-  else
-    hipLaunchKernelGGL((gemm_kernel<S, false>), grid, dim3(G_NT), 0, stream, p, vec);
+    return;
+  }
+  if constexpr (S != ANIMA_STORAGE_FP16) {
+    if (gemm_quad(p, S)) {
+      hipLaunchKernelGGL((gemm_kernel<S, false, true>), grid, dim3(G_NT), 0, stream, p, vec);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((gemm_kernel<S, false>), grid, dim3(G_NT), 0, stream, p, vec);
 }
 
 void launch_gemm(const GemmParams& p, int storage, hipStream_t stream) {
