@@ -617,14 +617,18 @@ constexpr int64_t F2_MIN_BLOCKS = 256;
 constexpr int F2_MIN_SPLIT_KEYS = 512;
 
 // Fine splits of the wide kernel (head_dim 384): one head has few query tiles, and a 32-key
-// tile costs a workgroup 1.7-2 us in series, so the call's time is its longest split.  Splits
+// tile costs a workgroup 1.6 us in series, so the call's time is its longest split.  Splits
 // down to 64 keys, 16 at most, as far as one round of workgroups goes; the splits' prologues
-// run beside each other.  us, 512-key splits -> fine: 378 tokens 27.9 -> 19.5, 792 48.5 ->
-// 25.7, 1215 43.5 -> 22.4, 1972 47.7 -> 28.6, 2808 44.7 -> 32.5, 3285 45.7 -> 38.0; 4096
-// tokens (32 tiles, 8 splits either way) 46.  Where 512-key splits leave one (fewer than
-// 1024 keys), the row stayed in fp32 registers: its partial rows are fp32 too.  Errors
-// against 64 bits: 2.96e-4 -> 2.76e-4 there, 3.61e-4 -> 3.56e-4 above.
+// run beside each other.  us, 512-key splits -> fine: 1215 tokens 43.5 -> 22.4, 1972 47.7 ->
+// 28.6, 2808 44.7 -> 32.5, 3285 45.7 -> 38.0; 4096 tokens (32 tiles, 8 splits either way) 46.
+// Where 512-key splits leave one (fewer than 1024 keys), the row stayed in fp32 registers: its
+// partial rows are fp32 too, and they and the merge cost 7.2 us and 0.65 ns a row, as much as
+// the key tiles they save in calls of few keys or many queries: the least of the sum is taken
+// (378 tokens 27.9 -> 19.5, 792 48.5 -> 25.7; 4096 queries to 500 keys 35.0 unsplit, 30.2 in
+// four, 40.9 in eight; 2048 to 100 15.8 unsplit, 21.1 in two).  Errors against 64 bits:
+// 2.96e-4 -> 2.76e-4 there, 3.61e-4 -> 3.56e-4 above.
 constexpr int FW_MIN_SPLIT_KEYS = 64;
+constexpr int64_t FW_CHUNK_PS = 2 * 1600000, FW_MERGE_PS = 7200000, FW_ROW_PS = 650;   // a chunk, a merge, a row of it
 
 static int coarse_kv_splits(const FlashParams& p, int D, int batch, int flash_rows) {
   if (p.causal || p.key_lengths_dev || p.use_host_lengths) return 1;
@@ -651,8 +655,23 @@ int flash_kv_splits(const FlashParams& p, int D, int batch, int flash_rows) {
   const int most = (int)std::min<int64_t>(F2_MIN_BLOCKS / tiles, FLASH_MAX_FINE_SPLITS);
   if (most <= coarse) return coarse;
   const int chunks = (p.Sk + FW_MIN_SPLIT_KEYS - 1) / FW_MIN_SPLIT_KEYS;
-  const int each = (chunks + most - 1) / most;
-  return std::max(coarse, (chunks + each - 1) / each);
+  if (coarse > 1) {
+    const int each = (chunks + most - 1) / most;
+    return std::max(coarse, (chunks + each - 1) / each);
+  }
+  const int64_t rows = (int64_t)p.Sq * p.H * batch;
+  int best = 1;
+  int64_t least = chunks * FW_CHUNK_PS;
+  for (int s = 2; s <= most && s <= chunks; ++s) {
+    const int each = (chunks + s - 1) / s;
+    if ((chunks + each - 1) / each != s) continue;   // the chunks fill fewer splits
+    const int64_t cost = each * FW_CHUNK_PS + FW_MERGE_PS + s * rows * FW_ROW_PS;
+    if (cost < least) {
+      least = cost;
+      best = s;
+    }
+  }
+  return best;
 }
 
 bool flash_split_f32(const FlashParams& p, int D, int batch, int flash_rows) {

@@ -80,3 +80,16 @@ def test_wide_noalloc_equals_encode_beyond_its_scratch(ctx):
     ex.encode_noalloc(output=outs[1], **args)
     torch.cuda.synchronize()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+# Calls whose fp32 partial rows cost more than the key tiles they would save, and one that splits.
+@pytest.mark.parametrize("H,Sq,Sk,splits", [(1, 4096, 100, 1), (1, 2048, 256, 1), (8, 1024, 192, 1), (1, 128, 128, 1),
+                                            (1, 4096, 500, 4), (2, 100, 1000, 16)])
+def test_wide_split_count(ctx, H, Sq, Sk, splits):
+    q, k, v = (torch.randn(H, n, D, device="cuda").half() for n in (Sq, Sk, Sk))
+    ex = AttentionExecutor(ctx, layout="headMajor")
+    print(f"WIDE COUNT H={H} Sq={Sq} Sk={Sk}", flush=True)
+    ex.execute(query=q, key=k, value=v, output=torch.empty_like(q), heads=H, query_count=Sq, key_count=Sk, head_dim=D)
+    rows = splits * H * Sq
+    need = (rows * D * 4 + 255) // 256 * 256 + rows * 8 if splits > 1 else 0
+    assert need <= ex.workspace_bytes() <= need + need // 8 + 8192
