@@ -130,9 +130,8 @@ void launch_gemm(const GemmParams& p, int storage, hipStream_t stream);
 // and weight rows, buffers below 2 GiB.  launch_gemm routes to it when it applies.
 bool pingpong_supported(const GemmParams& p, int storage);
 void launch_pingpong(const GemmParams& p, int storage, hipStream_t stream);
-// Its 128 x 256 tiles, and how many fill half the chip.
+// Its 128 x 256 tiles.
 inline int64_t pingpong_tiles(const GemmParams& p) { return (int64_t)((p.M + 127) / 128) * ((p.N + 255) / 256); }
-constexpr int64_t PG_FILL = 128;
 // Output rows over the input's: right where one workgroup reads all of X before it writes, as in
 // a ping-pong launch of one tile.  Such a linear is left to that kernel.
 inline bool single_tile_over_input(const GemmParams& p) {
@@ -152,12 +151,15 @@ bool pingpong_msplit(const GemmParams& p, int storage);
 // group and with a fused output stage.
 bool tile_preferred(const GemmParams& p, int storage);
 int tile_shape(const GemmParams& p);
+// The same two for one launch of several problems.
+bool tile_group_preferred(const GemmParams* ps, int count);
+int tile_group_shape(const GemmParams* ps, int count);
 // K splits of a single launch: the caller passes p.part = [splits][M][N] fp32 and p.ksplit.
 int tile_ksplit(const GemmParams& p);
 // Whether the problem's tile holds whole 128-column heads (GEMM_QK_NORM).
 bool tile_takes_norm(const GemmParams& p);
-// count (1..PG_GROUP) problems of one K, storage and tile shape in one launch.
-void launch_tile_group(const GemmParams* ps, int count, int storage, hipStream_t stream);
+// count (1..PG_GROUP) problems of one K and storage in one launch of tiles of one shape.
+void launch_tile_group(const GemmParams* ps, int count, int storage, int shape, hipStream_t stream);
 // The gated MLP in one launch: y = half(silu(half(X gate^T)) * half(X up^T)) into ps[0].y, for
 // ps[0] the gate and ps[1] the up projection of one input, shape and row stride.
 bool gated_pair_supported(const GemmParams* ps, int storage);
@@ -207,15 +209,15 @@ class LinearExecutor {
   bool encode_fused(anima_buffer input, int64_t input_offset, const anima_qweight& weight, anima_buffer output,
                     int64_t output_offset, int64_t input_rows, int32_t family, int epilogue, float* residual,
                     const float* gate);
-  // count (1..PG_GROUP) linears of one input, each into its own output, as one
-  // launch when every one of them takes the same tiled kernel (same K, storage and tile);
-  // otherwise encode() for each in turn.
+  // count (1..PG_GROUP) linears of one input, each into its own output: the members that
+  // encode() would run in one tiled kernel (same K, storage and tile shape) as one launch,
+  // encode() for the others.
   // With epi (one per weight): the output stages run in the GEMM and encode_group
   // returns true; if the group cannot run as one launch it encodes nothing
   // and returns false.  Without epi it always encodes and returns true.
-  // one_launch: members that would each take the small tiles run as one ping-pong launch
-  // when together they fill half the chip with its tiles, and members of up to 64 rows as one
-  // launch of the small tiles; their bits are then those of that kernel, not of a separate
+  // one_launch: members that would each take the small tiles run as one launch, of these tiles
+  // where one round holds them all, else of the ping-pong kernel's; so do members of up to 64
+  // rows.  Their bits are then those of that kernel and shape, not of a separate
   // encode() (block.hip, where nothing compares).
   bool encode_group(anima_buffer input, const anima_qweight* const* weights, const anima_buffer* outputs, int count,
                     int64_t input_rows, int32_t family, const GemmEpilogueArgs* epi = nullptr,

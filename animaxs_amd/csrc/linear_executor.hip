@@ -140,60 +140,73 @@ bool LinearExecutor::encode_group(anima_buffer input, const anima_qweight* const
     fail(ANIMA_E_INVALID_ARGUMENT, "unknown linear family");
   if (!(input_rows > 0)) fail(ANIMA_E_INVALID_SHAPE, "invalid LinearExecutor shape or offset");
   GemmParams ps[PG_GROUP];
-  int storage = -1, small_tiles = 0;
-  int64_t tiles = 0;
-  // together: one launch of one tiled kernel.  same_bits: a member that encode() would run
-  // in another form (split over K, small tiles, another tile shape or the M-split form)
-  // runs on its own instead, so that the bits match encode().
-  bool together = cfg_.backend == ANIMA_LINEAR_BACKEND_AUTO, same_bits = true;
+  int storage[PG_GROUP], kernel[PG_GROUP];   // the tiled kernel of encode(): 0 ping-pong, 1 + shape small tiles
+  // tiled: one launch can hold it.  same_bits: with the bits of encode(), that is, encode()
+  // runs it in a form that groups have (neither split over K nor in the M-split form; a
+  // linear alone keeps these here too, but split sums take no Q/K norm).
+  bool tiled[PG_GROUP], same_bits[PG_GROUP], any_small = false, any_split = false, all = true;
   for (int i = 0; i < count; ++i) {
     const QWeightView w = validate_weight(*weights[i], "LinearExecutor");
     ps[i] = prepare(input, 0, w, outputs[i], 0, input_rows);
+    storage[i] = w.storage;
     // Up to 64 rows a single linear streams its weights in another kernel; one launch of the
     // small tiles is still faster than two or three of those (encoder layer of 8 / 40 / 62
     // tokens, Q, K and V together: 57.5 -> 48.5, 66.4 -> 52.8, 72.4 -> 56.2 us).
-    together = together && (one_launch || !smallm_preferred(ps[i], w.storage)) && pingpong_supported(ps[i], w.storage) &&
-               (i == 0 || (w.storage == storage && ps[i].K == ps[0].K));
-    storage = w.storage;
-    if (!together) continue;
-    const bool small = tile_preferred(ps[i], storage), norm = epi && epi[i].epilogue == GEMM_QK_NORM;
-    small_tiles += small ? 1 : 0;
-    tiles += pingpong_tiles(ps[i]);
-    // Alone, a linear keeps its split or its M-split form here; split sums take no Q/K norm.
-    same_bits = same_bits && (small ? (count == 1 && !norm) || tile_ksplit(ps[i]) == 1
-                                    : count == 1 || !pingpong_msplit(ps[i], storage)) &&
-                (!small || tile_shape(ps[i]) == tile_shape(ps[0]));
+    tiled[i] = cfg_.backend == ANIMA_LINEAR_BACKEND_AUTO && (one_launch || !smallm_preferred(ps[i], w.storage)) &&
+               pingpong_supported(ps[i], w.storage);
+    const bool small = tiled[i] && tile_preferred(ps[i], w.storage), norm = epi && epi[i].epilogue == GEMM_QK_NORM;
+    const bool split = small && tile_ksplit(ps[i]) > 1;
+    kernel[i] = small ? 1 + tile_shape(ps[i]) : 0;
+    same_bits[i] = tiled[i] && (small ? !split || (count == 1 && !norm) : count == 1 || !pingpong_msplit(ps[i], w.storage));
+    any_small = any_small || small;
+    any_split = any_split || split;
+    all = all && tiled[i] && storage[i] == storage[0] && ps[i].K == ps[0].K;
   }
-  // Small tiles pay several rounds where one of 128 x 256 tiles would do.
-  const bool merged = one_launch && small_tiles > 0 && count > 1 && tiles >= PG_FILL;
-  if (merged)
-    small_tiles = 0;
-  else
-    together = together && same_bits && (small_tiles == 0 || small_tiles == count);
+  DeviceGuard guard(ctx_);
+  auto launch = [&](const GemmParams* qs, int n, int which, int st) {
+    if (which > 0)
+      launch_tile_group(qs, n, st, which - 1, ctx_->stream);
+    else
+      launch_pingpong_group(qs, n, st, ctx_->stream);
+  };
   if (epi) {
     for (int i = 0; i < count; ++i) {
       if (epi[i].epilogue != GEMM_STORE && epi[i].epilogue != GEMM_QK_NORM)
         fail(ANIMA_E_INVALID_ARGUMENT, "grouped linears take plain or Q/K-norm output stages");
+      all = all && same_bits[i] && kernel[i] == kernel[0];
       if (epi[i].epilogue == GEMM_QK_NORM) {
-        together = together && epi[i].norm_w && aligned16(epi[i].norm_w) && ps[i].N % 128 == 0 &&
-                   (small_tiles == 0 || tile_takes_norm(ps[i]));
+        all = all && epi[i].norm_w && aligned16(epi[i].norm_w) && ps[i].N % 128 == 0 &&
+              (kernel[i] == 0 || tile_takes_norm(ps[i]));
         ps[i].epilogue = GEMM_QK_NORM;
         ps[i].norm_w = epi[i].norm_w;
         ps[i].eps = epi[i].eps;
       }
     }
-    if (!together) return false;
-  }
-  if (!together) {
-    for (int i = 0; i < count; ++i) encode(input, 0, *weights[i], outputs[i], 0, input_rows, family);
+    if (!all) return false;
+    if (count == 1) plan_tile_splits(ps[0], storage[0], ctx_->stream);
+    launch(ps, count, kernel[0], storage[0]);
     return true;
   }
-  DeviceGuard guard(ctx_);
-  if (count == 1) plan_tile_splits(ps[0], storage, ctx_->stream);
-  if (small_tiles)
-    launch_tile_group(ps, count, storage, ctx_->stream);
-  else
-    launch_pingpong_group(ps, count, storage, ctx_->stream);
+  // Small tiles pay several rounds where one of 128 x 256 tiles would do.
+  if (one_launch && all && count > 1 && any_small && !any_split) {
+    launch(ps, count, tile_group_preferred(ps, count) ? 1 + tile_group_shape(ps, count) : 0, storage[0]);
+    return true;
+  }
+  bool done[PG_GROUP] = {};
+  for (int i = 0; i < count; ++i) {
+    if (done[i]) continue;
+    GemmParams qs[PG_GROUP];
+    int n = 0;
+    for (int j = i; j < count; ++j)
+      if (same_bits[i] && same_bits[j] && !done[j] && kernel[j] == kernel[i] && storage[j] == storage[i] && ps[j].K == ps[i].K) {
+        qs[n++] = ps[j];
+        done[j] = true;
+      }
+    if (n > 1)
+      launch(qs, n, kernel[i], storage[i]);
+    else
+      encode(input, 0, *weights[i], outputs[i], 0, input_rows, family);
+  }
   return true;
 }
 

@@ -1,5 +1,5 @@
 // Quantized GEMM on small tiles for gfx950: Y[M,N] = X[M,K] deq(W)[N,K]^T for W4/W8
-// weights where 128 x 256 tiles (linear_pingpong.hip) leave half of the chip idle: a
+// weights where 128 x 256 tiles (linear_pingpong.hip) leave most of the chip idle: a
 // prompt's rows, a 512-pixel image's tokens, the context projections.
 //
 //   * Tile TM x TN = (32 MT) x (32 WN), computed as C^T = W X^T on v_mfma_f32_32x32x16_f16
@@ -415,12 +415,23 @@ static int64_t tile_count(const GemmParams& p, int shape) {
 // 64 M=1024 N=2048 K=2048 17.3 / 29.4.
 bool tile_preferred(const GemmParams& p, int storage) {
   if (!pingpong_supported(p, storage) || single_tile_over_input(p)) return false;
-  return pingpong_tiles(p) < PG_FILL;
+  return pingpong_tiles(p) < 128;
 }
 
-int tile_shape(const GemmParams& p) {
-  return tile_count(p, 1) <= 256 ? 1 : 0;
+// One launch of several plain linears: where one round of tiles holds them.
+bool tile_group_preferred(const GemmParams* ps, int count) {
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += tile_count(ps[i], 0);
+  return tiles <= 256;
 }
+
+int tile_group_shape(const GemmParams* ps, int count) {
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += tile_count(ps[i], 1);
+  return tiles <= 256 ? 1 : 0;
+}
+
+int tile_shape(const GemmParams& p) { return tile_group_shape(&p, 1); }
 
 bool tile_takes_norm(const GemmParams& p) { return TG_TN[tile_shape(p)] % 128 == 0; }
 
@@ -473,21 +484,19 @@ static bool tile_swin(const GemmParams& p, int shape) {
          (reinterpret_cast<uintptr_t>(p.zero) & (piece - 1)) == 0;
 }
 
-void launch_tile_group(const GemmParams* ps, int count, int storage, hipStream_t stream) {
+void launch_tile_group(const GemmParams* ps, int count, int storage, int shape, hipStream_t stream) {
   if (count < 1 || count > PG_GROUP) fail(ANIMA_E_INVALID_ARGUMENT, "tiled GEMM group holds 1 to 3 problems");
   GemmGroup g{};
   bool swin = true;
-  const int shape = tile_shape(ps[0]);
   int64_t tiles = 0;
   for (int i = 0; i < count; ++i) {
     const GemmParams& p = ps[i];
     if (!pingpong_supported(p, storage)) fail(ANIMA_E_INVALID_SHAPE, "tiled GEMM: unsupported shape or alignment");
-    if (p.K != ps[0].K || tile_shape(p) != shape)
-      fail(ANIMA_E_INVALID_SHAPE, "tiled GEMM group: problems must share K and tile shape");
+    if (p.K != ps[0].K) fail(ANIMA_E_INVALID_SHAPE, "tiled GEMM group: problems must share K");
     check_gemm_epilogue(p);
     if (p.epilogue == GEMM_QK_NORM && TG_TN[shape] % 128 != 0)
       fail(ANIMA_E_INVALID_ARGUMENT, "GEMM Q/K-norm epilogue needs whole heads in a tile");
-    if (p.ksplit > 1 && (count != 1 || !p.part || p.ksplit != tile_ksplit(p)))
+    if (p.ksplit > 1 && (count != 1 || !p.part || shape != tile_shape(p) || p.ksplit != tile_ksplit(p)))
       fail(ANIMA_E_INVALID_ARGUMENT, "tiled GEMM: split K needs a single GEMM and its partial buffer");
     swin = swin && tile_swin(p, shape);
     g.p[i] = p;
@@ -508,8 +517,8 @@ bool gated_pair_supported(const GemmParams* ps, int storage) {
          ps[0].N <= 0x7fffffff - 256;
 }
 
-// The ping-pong kernel from half a chip of its 128-row tiles (128 columns of each member),
-// as for a group; below it 32-row tiles where one round holds them, else 64-row ones
+// The ping-pong kernel from half a chip of its 128-row tiles (128 columns of each member);
+// below it 32-row tiles where one round holds them, else 64-row ones
 // (two rounds of 32-row tiles cost a layer of 77 tokens 63.7 us against 60.0, of 250 84.3
 // against 73.9).  Gate, up and product against two launches, encoder layer, us: 77 tokens 63.7
 // -> 59.7, 4 x 512 166.1 -> 161.7, 344 x 2 120.1 -> 117.4.
@@ -519,7 +528,7 @@ void launch_gated_pair(const GemmParams* ps, int storage, hipStream_t stream) {
     fail(ANIMA_E_INVALID_ARGUMENT, "gated pair: no other output stage and no split K");
   const GemmParams& p = ps[0];
   auto count = [&](int tm, int tn) { return (int64_t)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn); };
-  if (count(128, 128) >= PG_FILL) {
+  if (count(128, 128) >= 128) {
     launch_pingpong_pair(ps, storage, stream);
     return;
   }
@@ -535,7 +544,7 @@ void launch_gated_pair(const GemmParams* ps, int storage, hipStream_t stream) {
 
 void launch_tiled(const GemmParams& p, int storage, hipStream_t stream) {
   if (tile_preferred(p, storage))
-    launch_tile_group(&p, 1, storage, stream);
+    launch_tile_group(&p, 1, storage, tile_shape(p), stream);
   else
     launch_pingpong(p, storage, stream);
 }

@@ -57,3 +57,47 @@ def test_small_m_past_the_streaming_limit(ctx, storage, M, N, K):
     torch.cuda.synchronize()
     for a, b in ((gelu, want), (r[0], r[1]), (r[2], r[3]), (group[0], branch), (group[1], branch)):
         assert torch.equal(_bits(a), _bits(b))
+
+
+# Members of the ping-pong kernel and of small tiles, of both tile shapes, one that splits K
+# between two that do not, two storages, and rows that fill the ping-pong kernel together.
+@pytest.mark.parametrize("M,members,K", [(2000, ((1, 2048), (1, 1024), (1, 1024)), 512),
+                                         (300, ((0, 2048), (0, 1024), (0, 1024)), 1024),
+                                         (77, ((1, 4096), (1, 256), (1, 4096)), 4096),
+                                         (512, ((0, 1024), (1, 1024), (0, 1024)), 512),
+                                         (2100, ((0, 1024), (0, 1024)), 512), (77, ((1, 192), (1, 64)), 192)])
+def test_groups_of_several_kernels(ctx, M, members, K):
+    qws = [_weight(st, N, K, i + N, False)[0] for i, (st, N) in enumerate(members)]
+    x = dev(torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half())
+    lin = LinearExecutor(ctx)
+    refs, outs = ([torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _, N in members]
+                  for _ in range(2))
+    print(f"GROUP KERNELS M={M} members={members} K={K}", flush=True)
+    for qw, r in zip(qws, refs):
+        lin.encode(x, qw, r, M)
+    lin.encode_group(x, qws, outs, M)
+    torch.cuda.synchronize()
+    for r, o in zip(refs, outs):
+        assert bool(torch.isfinite(r).all()) and torch.equal(_bits(r), _bits(o))
+
+
+# Encoder layers whose Q, K and V are one launch: of small tiles of one shape where the linears
+# alone would take two, of the narrow ones, and of the ping-pong kernel in place of small tiles.
+@pytest.mark.parametrize("S", [20, 150, 300, 700])
+def test_encoder_projections_in_one_launch(ctx, S):
+    from animaxs_amd import QwenLayerExecutor
+    from oracle import blocks, inputs
+    from tests.helpers import device_weight, mean_rel
+    d = inputs.qwen_layer(B=1, S=S, hidden=256, heads=16, kv_heads=8, intermediate=192)
+    print(f"ENCODER S={S}", flush=True)
+    weights, keep = {}, []
+    for n, w in d["w"].items():
+        weights[n], k = device_weight(w)
+        keep.append(k)
+    norms = {n: dev(d[n]) for n in ("input_norm", "post_attention_norm", "q_norm", "k_norm")}
+    residual = dev(d["x"].clone())
+    QwenLayerExecutor(ctx).encode(weights, norms, residual, dev(d["rope"]), batch=1, tokens=S,
+                                  key_lengths=d["key_lengths"].numpy(), hidden=256, heads=16, kv_heads=8, intermediate=192)
+    torch.cuda.synchronize()
+    ref = blocks.qwen_layer(d, boundary="fp16") - d["x"]
+    assert mean_rel(residual.cpu() - d["x"], ref) <= 2e-3
