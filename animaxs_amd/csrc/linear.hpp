@@ -27,7 +27,7 @@ struct GemmParams {
   int epilogue;
   float* residual;        // [M, N] fp32, GEMM_GATE_ADD / GEMM_RESIDUAL_ADD
   const float* gate;      // [N] fp32, GEMM_GATE_ADD
-  // Split K (small-tile and small-M kernels, single problem): ksplit workgroups per tile
+  // Split K (tiled and small-M kernels, single problem): ksplit workgroups per tile
   // each sum K / ksplit and write fp32 rows to part [ksplit][M][N]; a second kernel adds
   // them in split order, rounds once and runs the output stage (not GEMM_QK_NORM).
   int ksplit;
@@ -130,8 +130,9 @@ void launch_gemm(const GemmParams& p, int storage, hipStream_t stream);
 // and weight rows, buffers below 2 GiB.  launch_gemm routes to it when it applies.
 bool pingpong_supported(const GemmParams& p, int storage);
 void launch_pingpong(const GemmParams& p, int storage, hipStream_t stream);
-// Its 128 x 256 tiles.
+// Its 128 x 256 tiles, and its K splits of a single launch (1: none; else as tile_ksplit's).
 inline int64_t pingpong_tiles(const GemmParams& p) { return (int64_t)((p.M + 127) / 128) * ((p.N + 255) / 256); }
+int pingpong_ksplit(const GemmParams& p, int storage);
 // Output rows over the input's: right where one workgroup reads all of X before it writes, as in
 // a ping-pong launch of one tile.  Such a linear is left to that kernel.
 inline bool single_tile_over_input(const GemmParams& p) {
@@ -165,6 +166,10 @@ void launch_tile_group(const GemmParams* ps, int count, int storage, int shape, 
 bool gated_pair_supported(const GemmParams* ps, int storage);
 void launch_gated_pair(const GemmParams* ps, int storage, hipStream_t stream);
 void launch_pingpong_pair(const GemmParams* ps, int storage, hipStream_t stream);
+// K splits of a single launch of the tiled kernel that the problem prefers.
+inline int tiled_ksplit(const GemmParams& p, int storage) {
+  return tile_preferred(p, storage) ? tile_ksplit(p) : pingpong_ksplit(p, storage);
+}
 // The small-tile kernel or the ping-pong kernel, whichever the problem prefers.
 void launch_tiled(const GemmParams& p, int storage, hipStream_t stream);
 
@@ -238,8 +243,8 @@ class LinearExecutor {
   anima_ctx* context() const { return ctx_; }
 
  private:
-  // The small-tile kernel's K splits of a single launch, with their partial rows.
-  void plan_tile_splits(GemmParams& p, int storage, hipStream_t stream);
+  // The tiled kernels' K splits of a single launch, with their partial rows.
+  void plan_splits(GemmParams& p, int storage, hipStream_t stream);
   GemmParams prepare(anima_buffer input, int64_t input_offset, const QWeightView& w, anima_buffer output,
                      int64_t output_offset, int64_t input_rows) const;
   anima_ctx* ctx_;

@@ -78,9 +78,8 @@ GemmParams LinearExecutor::prepare(anima_buffer input, int64_t input_offset, con
   return p;
 }
 
-void LinearExecutor::plan_tile_splits(GemmParams& p, int storage, hipStream_t stream) {
-  if (!tile_preferred(p, storage)) return;
-  const int ks = tile_ksplit(p);
+void LinearExecutor::plan_splits(GemmParams& p, int storage, hipStream_t stream) {
+  const int ks = tiled_ksplit(p, storage);
   if (ks == 1) return;
   const int64_t bytes = checked_product({(int64_t)ks, p.M, p.N, 4}, "LinearExecutor");
   if (!ws_.available(bytes, stream)) return;   // a first call under capture runs unsplit
@@ -128,7 +127,7 @@ void LinearExecutor::encode(anima_buffer input, int64_t input_offset, const anim
     launch_smallm(p, w.storage, stream);
     return;
   }
-  plan_tile_splits(p, w.storage, stream);
+  plan_splits(p, w.storage, stream);
   launch_gemm(p, w.storage, stream);
 }
 
@@ -155,9 +154,9 @@ bool LinearExecutor::encode_group(anima_buffer input, const anima_qweight* const
     tiled[i] = cfg_.backend == ANIMA_LINEAR_BACKEND_AUTO && (one_launch || !smallm_preferred(ps[i], w.storage)) &&
                pingpong_supported(ps[i], w.storage);
     const bool small = tiled[i] && tile_preferred(ps[i], w.storage), norm = epi && epi[i].epilogue == GEMM_QK_NORM;
-    const bool split = small && tile_ksplit(ps[i]) > 1;
+    const bool split = tiled[i] && tiled_ksplit(ps[i], w.storage) > 1;
     kernel[i] = small ? 1 + tile_shape(ps[i]) : 0;
-    same_bits[i] = tiled[i] && (small ? !split || (count == 1 && !norm) : count == 1 || !pingpong_msplit(ps[i], w.storage));
+    same_bits[i] = tiled[i] && (!split || (count == 1 && !norm)) && (count == 1 || !pingpong_msplit(ps[i], w.storage));
     any_small = any_small || small;
     any_split = any_split || split;
     all = all && tiled[i] && storage[i] == storage[0] && ps[i].K == ps[0].K;
@@ -183,7 +182,7 @@ bool LinearExecutor::encode_group(anima_buffer input, const anima_qweight* const
       }
     }
     if (!all) return false;
-    if (count == 1) plan_tile_splits(ps[0], storage[0], ctx_->stream);
+    if (count == 1) plan_splits(ps[0], storage[0], ctx_->stream);
     launch(ps, count, kernel[0], storage[0]);
     return true;
   }
@@ -228,7 +227,7 @@ bool LinearExecutor::encode_fused(anima_buffer input, int64_t input_offset, cons
   p.gate = gate;
   DeviceGuard guard(ctx_);
   // The split decision is the one encode() makes, so the bits match encode() + the step.
-  plan_tile_splits(p, w.storage, ctx_->stream);
+  plan_splits(p, w.storage, ctx_->stream);
   launch_tiled(p, w.storage, ctx_->stream);
   return true;
 }

@@ -120,7 +120,11 @@ void pingpong_gemm_kernel(GemmGroup gp) {
   const int wrow = 64 * (PAIR ? wg & 1 : wg);        // and its first row in the tile
   const int vec_store = gp.vec[pi];
   const int ntn = (p.N + BN - 1) / BN;
-  const int lt = lbg - gp.first_tile[pi];
+  // Split K (single launches of the K-split form): workgroup lb takes K-block range `split` of
+  // tile lb / ks.
+  const int lb = lbg - gp.first_tile[pi];
+  const int ks = MSPLIT || PAIR || p.ksplit <= 1 ? 1 : p.ksplit;
+  const int split = lb % ks, lt = lb / ks;
   // Tiles go in groups of PG_GM M blocks x all N tiles, M varying fastest: the 32
   // consecutive tiles an XCD runs in one round are 4 M blocks x 8 N tiles, so each weight
   // tile it loads serves four workgroups from its L2 (N varying fastest, a round of a wide
@@ -131,7 +135,7 @@ void pingpong_gemm_kernel(GemmGroup gp) {
   const int gr = lt % (GM * ntn);
   const int tm = gfirst + gr % gm, tn = gr / gm;
   const int m0 = tm * BM, n0 = tn * BN;
-  const int nk = p.K / PG_BK;
+  const int nk = p.K / PG_BK / ks, kbeg = split * nk;
   // Group 0 takes K blocks [0, half), group 1 [half, nk); with windows, half is a
   // multiple of the window so every window is aligned.
   int half = SWIN ? PG_WIN * ((nk + 2 * PG_WIN - 1) / (2 * PG_WIN)) : (nk + 1) / 2;
@@ -140,17 +144,18 @@ void pingpong_gemm_kernel(GemmGroup gp) {
   const int nown = MSPLIT ? nk : (group == 0 ? half : nk - half);
 
   // Tile-relative buffers (sizes fit in 31 bits; checked on the host).
+  // With split K they start at the split's first K block; the sizes end where they did.
   // The group's X rows start at xr0 (M-split: its 128-row half of the tile, which can
   // lie past M on the last tile row: then the descriptor is empty and reads zeros).
   const int xr0 = m0 + (MSPLIT ? PG_BM * group : 0);
-  const half_t* xb = p.x + (int64_t)xr0 * p.K;
-  const int xrem = (p.M - xr0) * p.K * 2;
+  const half_t* xb = p.x + (int64_t)xr0 * p.K + kbeg * PG_BK;
+  const int xrem = (p.M - xr0) * p.K * 2 - kbeg * PG_BK * 2;
   const int xbytes = xrem > 0 ? xrem : 0;
-  const uint8_t* wb = pw.w + (int64_t)n0 * p.row_stride;
-  const int wbytes = (int)((int64_t)(p.N - n0) * p.row_stride);
-  const half_t* sb = pw.scale + (int64_t)n0 * p.groups;
-  const half_t* zb = pw.zero + (int64_t)n0 * p.groups;
-  const int sbytes = (p.N - n0) * p.groups * 2;
+  const uint8_t* wb = pw.w + (int64_t)n0 * p.row_stride + kbeg * 32 * WCH;
+  const int wbytes = (int)((int64_t)(p.N - n0) * p.row_stride) - kbeg * 32 * WCH;
+  const half_t* sb = pw.scale + (int64_t)n0 * p.groups + kbeg;
+  const half_t* zb = pw.zero + (int64_t)n0 * p.groups + kbeg;
+  const int sbytes = (p.N - n0) * p.groups * 2 - kbeg * 2;
 
   // X copies: thread t of a group moves chunks t + 256r (r < 4) of its group's
   // block: row t/8 + 32r, 16-byte column t%8 (8 lanes read one 128-byte row).
@@ -439,6 +444,33 @@ void pingpong_gemm_kernel(GemmGroup gp) {
           *reinterpret_cast<floatx4*>(own + (((t * 2 + j) * 4 + q) * 64 + lane) * 16) = v;
         }
     barrier();
+    if (ks > 1) {
+      // Split K: the fp32 sums of this K range go to the split's partial rows.
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int m = m0 + 32 * (MINE + j) + c32;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const floatx4 o = *reinterpret_cast<const floatx4*>(partner + (((t * 2 + j) * 4 + q) * 64 + lane) * 16);
+            const floatx4 sv = {acc[t][MINE + j][4 * q] + o[0], acc[t][MINE + j][4 * q + 1] + o[1],
+                                acc[t][MINE + j][4 * q + 2] + o[2], acc[t][MINE + j][4 * q + 3] + o[3]};
+            const int n = n0 + 64 * wg + 32 * t + 8 * q + 4 * hh;
+            if (m < p.M) {
+              float* prow = p.part + ((int64_t)split * p.M + m) * p.N;
+              if ((p.N & 3) == 0 && n + 3 < p.N) {
+                *reinterpret_cast<floatx4*>(prow + n) = sv;
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  if (n + e < p.N) prow[n + e] = sv[e];
+              }
+            }
+          }
+        }
+      return;
+    }
     half4v out[2][2][4];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -482,6 +514,7 @@ void pingpong_gemm_kernel(GemmGroup gp) {
       finish(std::integral_constant<int, 0>{});
     else
       finish(std::integral_constant<int, 2>{});
+    if (ks > 1) return;   // partial rows written; splitk_reduce_kernel finishes
   }
   barrier();
 
@@ -565,6 +598,24 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
+// K splits of a plain or fused launch whose 128-row tiles fill less than half the chip and
+// which the small tiles do not take: as many splits of >= 16 K blocks as keep the grid within
+// 256 workgroups (shorter splits lose more to the partial rows than they gain).  W8 M=1300
+// N=2048 K=4096: 45 us, 53 unsplit, 53 on the small tiles.
+int pingpong_ksplit(const GemmParams& p, int storage) {
+  if (!pingpong_supported(p, storage) || tile_preferred(p, storage)) return 1;
+  const int64_t tiles = pingpong_tiles(p);
+  if (tiles >= 128) return 1;
+  const int nk = p.K / PG_BK;
+  const bool swin = p.groups % PG_WIN == 0 && aligned16(p.scale) && aligned16(p.zero);
+  int best = 1;
+  for (int k = 2; k <= 8; ++k) {
+    if (nk % k != 0 || nk / k < 16 || (swin && (nk / k) % PG_WIN != 0) || tiles * k > 256) continue;
+    best = k;
+  }
+  return best;
+}
+
 // A single launch of p takes the M-split form when its 256-row tiles still fill at least
 // two whole rounds of the chip (512 workgroups): it then pays half as many first loads
 // and output stages per output, and no partial-sum exchange.  Fewer tiles would leave
@@ -596,11 +647,12 @@ void launch_pingpong_group(const GemmParams* ps, int count, int storage, hipStre
     if (p.K != ps[0].K) fail(ANIMA_E_INVALID_SHAPE, "ping-pong GEMM group: problems must share K");
     check_gemm_epilogue(p);
     swin = swin && p.groups % PG_WIN == 0 && aligned16(p.scale) && aligned16(p.zero);
-    if (p.ksplit > 1) fail(ANIMA_E_INVALID_ARGUMENT, "ping-pong GEMM: no split K");
+    if (p.ksplit > 1 && (count != 1 || !p.part || p.ksplit != pingpong_ksplit(p, storage)))
+      fail(ANIMA_E_INVALID_ARGUMENT, "ping-pong GEMM: split K needs a single GEMM and its partial buffer");
     g.p[i] = p;
     g.first_tile[i] = (int)tiles;
     g.vec[i] = gemm_vec_output(p);
-    tiles += (int64_t)((p.M + bm - 1) / bm) * ((p.N + PG_BN - 1) / PG_BN);
+    tiles += (int64_t)((p.M + bm - 1) / bm) * ((p.N + PG_BN - 1) / PG_BN) * (p.ksplit > 1 ? p.ksplit : 1);
     if (tiles > 0x7fffffff) fail(ANIMA_E_INVALID_SHAPE, "GEMM grid too large");
   }
   for (int i = count; i < PG_GROUP; ++i) g.first_tile[i] = (int)tiles;
@@ -618,6 +670,7 @@ void launch_pingpong_group(const GemmParams* ps, int count, int storage, hipStre
       launch_pingpong_t<ANIMA_STORAGE_W8, false>(g, tiles, msplit, stream);
   }
   ANIMA_HIP(hipGetLastError());
+  if (ps[0].ksplit > 1) launch_splitk_epilogue(ps[0], stream);
 }
 
 void launch_pingpong_pair(const GemmParams* ps, int storage, hipStream_t stream) {

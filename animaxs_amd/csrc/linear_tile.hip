@@ -409,13 +409,18 @@ static int64_t tile_count(const GemmParams& p, int shape) {
   return (int64_t)((p.M + TG_TM[shape] - 1) / TG_TM[shape]) * ((p.N + TG_TN[shape] - 1) / TG_TN[shape]);
 }
 
-// Below half a chip of 128 x 256 tiles.  At 128 of them the kernels meet (us, this / ping-
-// pong): M=2048 N=2048 K=2048 30.0 / 29.2-31.5, M=512 N=8192 K=2048 29.5-35 / 29.2-35.2,
-// M=4096 N=1024 K=2048 33.6-35 / 29-31.5; at 96 M=1024 N=3072 K=1024 18.7-20.2 / 18.7-20.0; at
-// 64 M=1024 N=2048 K=2048 17.3 / 29.4.
+// One round of 64 x 128 tiles (a quarter of a chip of 128 x 256 ones) takes 1/1.5 to 1/3.4 of
+// the ping-pong kernel's time: M=1024 N=2048 K=2048, 256 tiles, 17.3 / 29.4 us.  Two rounds,
+// below half a chip of the other's tiles, only at K = 512 and 1280 to 2048 in whole K blocks
+// (ping-pong / this over 288 to 512 tiles: plain 0.96-1.04 at 512, 1.03-1.11 at 1536, 0.94-1.07
+// at 2048; GELU 1.12-1.19, 1.06-1.19, 1.04-1.11; gate-add 1.04-1.10, 1.00-1.17, 0.94-1.10).
+// At 768 and 1024 the ping-pong kernel's halves of K are one window each (plain 0.91-1.00), at
+// 256 a block cannot hide the loads (0.86-0.93), a last block of one group costs a whole one
+// (320 0.70-0.74, 1088 0.74-0.77), and past 2048 the ping-pong kernel splits K (4096 0.83-0.96).
 bool tile_preferred(const GemmParams& p, int storage) {
   if (!pingpong_supported(p, storage) || single_tile_over_input(p)) return false;
-  return pingpong_tiles(p) < 128;
+  const bool two_rounds = p.K % 256 == 0 && (p.K == 512 || (p.K > 1024 && p.K <= 2048));
+  return tile_count(p, 0) <= 256 || (two_rounds && pingpong_tiles(p) < 128);
 }
 
 // One launch of several plain linears: where one round of tiles holds them.

@@ -60,12 +60,12 @@ def test_small_m_past_the_streaming_limit(ctx, storage, M, N, K):
 
 
 # Members of the ping-pong kernel and of small tiles, of both tile shapes, one that splits K
-# between two that do not, two storages, and rows that fill the ping-pong kernel together.
+# between two that do not, two storages, two rounds of tiles and the K that leaves them, and rows that fill the ping-pong kernel together.
 @pytest.mark.parametrize("M,members,K", [(2000, ((1, 2048), (1, 1024), (1, 1024)), 512),
                                          (300, ((0, 2048), (0, 1024), (0, 1024)), 1024),
                                          (77, ((1, 4096), (1, 256), (1, 4096)), 4096),
                                          (512, ((0, 1024), (1, 1024), (0, 1024)), 512),
-                                         (2100, ((0, 1024), (0, 1024)), 512), (77, ((1, 192), (1, 64)), 192)])
+                                         (2100, ((0, 1024), (0, 1024)), 512), (2100, ((0, 1024), (1, 1024)), 1024), (77, ((1, 192), (1, 64)), 192)])
 def test_groups_of_several_kernels(ctx, M, members, K):
     qws = [_weight(st, N, K, i + N, False)[0] for i, (st, N) in enumerate(members)]
     x = dev(torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half())
