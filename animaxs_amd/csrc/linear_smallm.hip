@@ -711,7 +711,12 @@ static int splitk_chunks(const GemmParams& p, int storage) {
   // of X (about 0.044 us per KB at 16-row blocks) costs more than the partial rows:
   // M=32 N=2048 K=4096 13.3 -> 8.5 us, M=16 K=8192 13.2 -> 10.9 us, M=8 K=16384
   // 17.4 -> 14.9 us; M=16 K=4096 ties and M=32 N=4096 K=2048 is 5 % slower split.
-  if (p.N >= 32 * 256 || (p.M <= 32 && (int64_t)p.M * p.K < 131072)) return 0;
+  // K = 64 (mod 128) streams with more rows too while X is up to 96 KB: one launch, as the
+  // tile kernels' before, where a group or a separate output stage has several of them (M=64
+  // N=1024 K=320 6.2 -> 3.8 us, M=48 N=6000 K=832 8.5 -> 7.0, M=33 N=2048 K=1344 7.0 -> 5.4).
+  if (p.N >= 32 * 256 || (p.M <= 32 && (int64_t)p.M * p.K < 131072) ||
+      (p.K % SM_CHUNK != 0 && (int64_t)p.M * p.K <= 49152))
+    return 0;
   if (p.M < 1 || p.M > SMALLM_MAX_ROWS || p.K < 1 || p.K % (SM_CHUNK / 2) != 0 || !aligned16(p.x) || !aligned16(p.w) ||
       p.row_stride % 16 != 0 || (int64_t)p.M * p.K * 2 > 0x7fffffff || (p.K % SM_CHUNK != 0 && single_tile_over_input(p)))
     return 0;

@@ -67,3 +67,11 @@ def test_infinite_last_group(ctx, storage, M, N, K):
     torch.cuda.synchronize()
     assert bool(torch.isposinf(y[:, 0]).all()) and bool(torch.isinf(dense[0, -64:]).all())
     assert bool(torch.isfinite(y[:, 1:]).all())
+
+
+# More than 32 rows on either side of the X that streams (96 KB) at K = 64 (mod 128).
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(33, 77, 1472), (33, 77, 1600), (48, 130, 960), (48, 130, 1088), (64, 300, 704),
+                                   (64, 300, 832), (64, 6000, 320)])
+def test_streamed_rows_limit(ctx, storage, M, N, K):
+    test_uneven_k(ctx, storage, M, N, K, 0)
