@@ -526,7 +526,8 @@ bool gated_pair_supported(const GemmParams* ps, int storage) {
 // below it 32-row tiles where one round holds them, else 64-row ones
 // (two rounds of 32-row tiles cost a layer of 77 tokens 63.7 us against 60.0, of 250 84.3
 // against 73.9).  Gate, up and product against two launches, encoder layer, us: 77 tokens 63.7
-// -> 59.7, 4 x 512 166.1 -> 161.7, 344 x 2 120.1 -> 117.4.
+// -> 59.7, 4 x 512 166.1 -> 161.7, 344 x 2 120.1 -> 117.4, with a cheaper SiLU than gated_silu8's,
+// which is 0.2 us of the first and 1.9 of the second.
 void launch_gated_pair(const GemmParams* ps, int storage, hipStream_t stream) {
   if (!gated_pair_supported(ps, storage)) fail(ANIMA_E_INVALID_SHAPE, "gated pair: unsupported shapes or alignment");
   if (ps[0].epilogue != GEMM_STORE || ps[0].ksplit > 1)

@@ -250,8 +250,8 @@ class LinearExecutor:
                                 _FAMILY[family]))
 
     def encode_group(self, input, weights, outputs, input_rows: int, family: str = "other") -> None:
-        """1..3 linears of one input, each into its own output (one launch when the tiled
-        GEMM takes them all)."""
+        """1..3 linears of one input, each into its own output, with the bits of separate encodes
+        (those that take the same tiled kernel share a launch)."""
         n = len(weights)
         if n != len(outputs):
             raise ValueError("weights and outputs differ in length")

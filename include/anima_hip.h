@@ -307,8 +307,8 @@ anima_status anima_linear_encode_epilogue(anima_linear* lin, anima_buffer input,
  * its own output -- the Q/K/V (or gate/up) projections that DiTBlockExecutor and
  * QwenEncoderMetal encode one after another on the same normalised input
  * (DiTBlockExecutor.swift:1035-1105, QwenEncoderMetal.swift:244-262).  Results equal
- * count anima_linear_encode calls bit for bit; when every weight takes the tiled
- * W4/W8 GEMM with the same K and storage, the linears run as one launch. */
+ * count anima_linear_encode calls bit for bit; weights that take the same tiled
+ * W4/W8 kernel, with the same K and storage, share a launch. */
 anima_status anima_linear_encode_group(anima_linear* lin, anima_buffer input, const anima_qweight* const* weights,
                                        const anima_buffer* outputs, int32_t count, int64_t input_rows,
                                        int32_t family);
